@@ -168,6 +168,42 @@ def test_gate_up_silu_every_gate(dev):
     assert bool(((got[:, 0].double() - exact).abs() <= ulp * (0.5 + 1e-3)).all())
 
 
+def test_gate_up_silu_bits(dev):
+    """act = fp16(g / (1 + exp(-g))) in fp32, bit for bit, for all 65536 fp16 gates:
+    finite ones, and infinite and NaN gates (which only the gate rows' scales make, so
+    that the up rows stay 1)."""
+    from lemoq import _hip
+
+    finite = torch.arange(0x7C00, dtype=torch.int32)
+    x0 = torch.cat((finite, finite | 0x8000)).to(torch.uint16).view(torch.float16)
+    T, H, F = int(x0.numel()), 64, 32
+    P, st = _hip.ptr, _hip.stream_of(dev)
+    x = torch.zeros((T, H), dtype=torch.float16)
+    x[:, 0], x[:, 1] = x0, 1.0
+    codes = torch.zeros((1, 2 * F, H), dtype=torch.int8)
+    codes[0, :F, 0] = 1  # gate rows pick x[0], up rows x[1]
+    codes[0, F:, 1] = 1
+    scale = torch.ones((1, 2 * F, 1), dtype=torch.float16)
+    codes[0, F - 2, 0], scale[0, F - 2, 0] = 127, 32768.0  # overflows to +-inf
+    scale[0, F - 1, 0] = float("nan")
+    i32 = dict(dtype=torch.int32, device=dev)
+    begins = torch.arange(0, T, 128)
+    tiles = torch.stack((torch.zeros_like(begins), begins, (begins + 128).clamp(max=T), torch.zeros_like(begins)), 1)
+    td = tiles.to(**i32).contiguous()
+    tok = torch.arange(T, **i32)
+    act = torch.empty((T, F), dtype=torch.float16, device=dev)
+    xd, cd, sd = x.to(dev), codes.to(dev), scale.to(dev)
+    _hip.call("lemoq_moe_prefill_gate_up", P(xd), H, P(tok), P(td), int(begins.numel()), P(cd), P(sd), F, 64,
+              P(act), st)
+    gates = torch.stack((xd[:, 0], (xd[:, 0].double() * (127 * 32768.0)).to(torch.float16), xd[:, 0] * float("nan")), 1)
+    g = gates.float()
+    want = (g / (1.0 + torch.exp(-g))).to(torch.float16)
+    got = act[:, F - 3:]
+    assert bool(gates.isinf().any()) and bool(gates.isnan().any())
+    same = (got.view(torch.int16) == want.view(torch.int16)) | (got.isnan() & want.isnan())
+    assert bool(same.all()), gates[~same].tolist()[:8]
+
+
 Q_CASES = [  # bits, symmetric, mxfp4, group
     (8, False, False, 32), (8, False, False, 128), (4, True, False, 32), (4, True, False, 96), (4, True, False, 128),
     (4, False, False, 64), (4, False, False, 128), (4, True, True, 32),
