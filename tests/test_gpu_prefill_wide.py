@@ -184,7 +184,7 @@ def test_gate_up_silu_bits(dev):
     codes[0, :F, 0] = 1  # gate rows pick x[0], up rows x[1]
     codes[0, F:, 1] = 1
     scale = torch.ones((1, 2 * F, 1), dtype=torch.float16)
-    codes[0, F - 2, 0], scale[0, F - 2, 0] = 127, 32768.0  # overflows to +-inf
+    codes[0, F - 2, 0], scale[0, F - 2, 0] = 127, 512.0  # gates beyond 1 overflow to +-inf
     scale[0, F - 1, 0] = float("nan")
     i32 = dict(dtype=torch.int32, device=dev)
     begins = torch.arange(0, T, 128)
@@ -195,7 +195,7 @@ def test_gate_up_silu_bits(dev):
     xd, cd, sd = x.to(dev), codes.to(dev), scale.to(dev)
     _hip.call("lemoq_moe_prefill_gate_up", P(xd), H, P(tok), P(td), int(begins.numel()), P(cd), P(sd), F, 64,
               P(act), st)
-    gates = torch.stack((xd[:, 0], (xd[:, 0].double() * (127 * 32768.0)).to(torch.float16), xd[:, 0] * float("nan")), 1)
+    gates = torch.stack((xd[:, 0], (xd[:, 0].double() * (127 * 512.0)).to(torch.float16), xd[:, 0] * float("nan")), 1)
     g = gates.float()
     want = (g / (1.0 + torch.exp(-g))).to(torch.float16)
     got = act[:, F - 3:]
