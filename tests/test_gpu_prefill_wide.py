@@ -159,7 +159,7 @@ def test_gate_up_silu_every_gate(dev):
     torch.cuda.synchronize()
     got = act.cpu()
     assert torch.equal(got, got[:, :1].expand_as(got))
-    g = gates.float()
+    g = gates.float() + 0.0  # a sum from 0 has no -0
     want = (g / (1.0 + torch.exp(-g))).to(torch.float16)
     off = (got[:, 0].view(torch.int16) != want.view(torch.int16)) & ~((got[:, 0] == 0) & (want == 0))
     exact = gates.double() / (1.0 + torch.exp(-gates.double()))
@@ -196,7 +196,7 @@ def test_gate_up_silu_bits(dev):
     _hip.call("lemoq_moe_prefill_gate_up", P(xd), H, P(tok), P(td), int(begins.numel()), P(cd), P(sd), F, 64,
               P(act), st)
     gates = torch.stack((xd[:, 0], (xd[:, 0].double() * (127 * 512.0)).to(torch.float16), xd[:, 0] * float("nan")), 1)
-    g = gates.float()
+    g = gates.float() + 0.0  # a sum from 0 has no -0
     want = (g / (1.0 + torch.exp(-g))).to(torch.float16)
     got = act[:, F - 3:]
     assert bool(gates.isinf().any()) and bool(gates.isnan().any())
