@@ -35,7 +35,7 @@
 // at T 5000 166 -> 157, 256 at T 4096 508 -> 474; the same bits.  Next tile's
 // scores under this tile's softmax needs more than 256 registers (T 4096: 150
 // us); eight waves with a key split of 4 is slower below T 300 and above T 1024.
-#include "common.h"
+#include "lds_dma.h"
 
 namespace {
 
@@ -76,11 +76,6 @@ struct AttnGeom {
   static_assert(PASSES >= 1 && KT % (RPL * NW) == 0, "tile split");
 };
 
-// LDS byte address of a shared array (also marks it as written by the direct
-// loads' asm, which the compiler cannot see into).
-typedef __attribute__((address_space(3))) uint8_t lds_byte;
-__device__ __forceinline__ uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)(const lds_byte*)p; }
-
 // The K and V rows [k0, k0 + KT) to an LDS buffer by direct loads, this wave's
 // share; rows past the prompt read its last row.
 template <class G>
@@ -97,11 +92,8 @@ __device__ __forceinline__ void attn_load(uint32_t buf, const uint16_t* __restri
     const uint32_t ko = (uint32_t)(src * G::ROW + (c ^ G::kswz(row)) * 16);
     const uint32_t vo = (uint32_t)(src * G::ROW + (c ^ G::vswz(row)) * 16);
     const uint32_t to = buf + (uint32_t)(first * G::ROW);
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(to), "v"(ko), "s"(kb) : "memory");
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(to + G::KB), "v"(vo), "s"(vb)
-                 : "memory");
+    dma16(to, ko, kb);
+    dma16(to + G::KB, vo, vb);
   }
 }
 

@@ -14,6 +14,7 @@
 #include <type_traits>
 
 #include "gemm_core.h"
+#include "lds_dma.h"
 
 namespace lemoq_gemm {
 
@@ -168,23 +169,6 @@ __device__ __forceinline__ uint32_t wide_c_chunk(int row, int lane) {
   return (uint32_t)(((lane % G::LPR) ^ wide_c_swizzle<G>(row)) * 16);
 }
 
-// LDS byte address of a shared array (also marks the array as written by the
-// direct loads' asm, which the compiler cannot see into).
-typedef __attribute__((address_space(3))) uint8_t lds_byte;
-__device__ __forceinline__ uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)(const lds_byte*)p; }
-
-// 64 lanes x 16 bytes from base + off (per lane) to LDS at `to` + 16 lane.
-// asm, because the compiler drains every direct load (vmcnt 0) before any LDS
-// read; the waits are wide_wait's.
-__device__ __forceinline__ void dma16(uint32_t to, uint32_t off, const uint8_t* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :
-               : "s"(to), "v"(off), "s"(base)
-               : "memory");
-}
-__device__ __forceinline__ void dma16(uint32_t to, uint64_t addr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(to), "v"(addr) : "memory");
-}
 // This wave's LDS reads are done and at most N of its direct loads are in
 // flight, in every wave of the block.
 template <int N>
