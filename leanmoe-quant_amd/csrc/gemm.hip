@@ -21,7 +21,6 @@
 // LDS and writes whole row segments in 16-byte chunks; otherwise each lane
 // stores its own elements.
 #include "gemm_wide.h"
-#include "row_gemm.h"
 
 #include <mutex>
 
@@ -265,22 +264,6 @@ __global__ __launch_bounds__(G::NT, 2) void gemm_q_kernel(const GemmArgs a) {
   }
 }
 
-// One row of int8 weights: a wave per 32 columns (row_gemm.h), the same bits.
-// The 64 x 128 tiles below leave most of the chip idle (16 blocks on 2048
-// columns) and pay 0.35 us a stage: ROWTIMES.
-__global__ __launch_bounds__(64) void gemm_w8_row_kernel(const GemmArgs a) {
-  __shared__ __align__(16) uint16_t xs[RowDot<true>::KB];
-  const int lane = threadIdx.x;
-  const int64_t n = (int64_t)blockIdx.x * RW_COLS + (lane & 31), row = n < a.N ? n : a.N - 1;
-  const int64_t m = a.x_rows ? (int64_t)a.x_rows[0] : 0;
-  RowDot<true> d(a.x + m * a.x_ld, reinterpret_cast<const int8_t*>(a.codes) + row * a.K,
-                 reinterpret_cast<const uint16_t*>(a.scale) + row * (a.K / a.group), (int)a.K, a.group);
-  uint16_t o = f2h(d.dot(xs));
-  if (lane >= 32 || n >= a.N) return;
-  if (a.resid) o = hadd_round(h2f(o), a.resid[n]);
-  a.y16[n] = o;
-}
-
 // Block shapes: two blocks per CU each (at most 80 KB of LDS).
 template <class Q>
 using QWide = WideGeo<Q, 4, 2, 4, 2, Q::ZERO ? 16 : 32>;   // 128 x 256
@@ -324,12 +307,6 @@ TilePick tile_pick(int64_t M, int64_t N, bool row_out) {
 
 template <class Q, bool GATHERS>
 int launch_q(GemmArgs a, hipStream_t st) {
-  if constexpr (std::is_same_v<Q, WideW8>) {
-    if (a.M == 1) {
-      hipLaunchKernelGGL(gemm_w8_row_kernel, dim3((unsigned)((a.N + RW_COLS - 1) / RW_COLS)), dim3(64), 0, st, a);
-      LEMOQ_CHECK_LAUNCH();
-    }
-  }
   const int64_t ng = a.K / a.group;
   a.scale_vec = !std::is_same_v<Q, WideMx4> && ng % 8 == 0 && lemoq_aligned16(a.scale);
   const TilePick pick = tile_pick(a.M, a.N, a.row_out != 0);
