@@ -297,12 +297,17 @@ int lemoq_moe_gate_up_w8_routed(const uint16_t* x, const int8_t* codes,
                                 int64_t ffn, int64_t hidden, int64_t group, uint16_t* act,
                                 int64_t* top_i, uint16_t* top_w, void* stream);
 
-/* lemoq_moe_gate_up_w8_routed and lemoq_moe_down_w8 with the arithmetic of the
- * multi-token block (_prefill_forward, src/lemoq/kernels/moe_static.py:329-371;
- * lemoq_moe_prefill_gate_up / _down / _combine): weights rounded to fp16 before
- * the dot, fp16 gate, up, silu and product, fp16 expert outputs times the fp16
- * routing weight, added in fp16 in ascending expert order.  For one row: the last
- * of a prefill. */
+/* lemoq_moe_gate_up_w8 / _routed and lemoq_moe_down_w8 with the arithmetic of
+ * the multi-token block (_prefill_forward, src/lemoq/kernels/moe_static.py:329-371;
+ * lemoq_moe_prefill_gate_up / _down / _combine, whose bits these give): weights
+ * rounded to fp16 before the dot, fp16 gate, up, silu and product, fp16 expert
+ * outputs times the fp16 routing weight, added in fp16 in ascending expert order.
+ * For one row: the last of a prefill.  lemoq_moe_gate_up_w8_dq takes the routing's
+ * ids and fp32 weights (lemoq_route_topk's) and rounds these to top_w. */
+int lemoq_moe_gate_up_w8_dq(const uint16_t* x, const int8_t* codes, const uint16_t* scale,
+                            const int64_t* ids, const float* top_w32, int64_t top_k,
+                            int64_t num_experts, int64_t ffn, int64_t hidden, int64_t group,
+                            uint16_t* act, uint16_t* top_w, void* stream);
 int lemoq_moe_gate_up_w8_routed_dq(const uint16_t* x, const int8_t* codes,
                                    const uint16_t* scale, const uint16_t* router_logits,
                                    int64_t top_k, int norm_topk_prob, int64_t num_experts,

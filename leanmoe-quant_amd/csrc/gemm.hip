@@ -21,6 +21,7 @@
 // LDS and writes whole row segments in 16-byte chunks; otherwise each lane
 // stores its own elements.
 #include "gemm_wide.h"
+#include "row_gemm.h"
 
 #include <mutex>
 
@@ -264,6 +265,30 @@ __global__ __launch_bounds__(G::NT, 2) void gemm_q_kernel(const GemmArgs a) {
   }
 }
 
+// One row of int8 weights: a wave per 32 columns (row_gemm.h), the same bits as
+// the tiles below, which for one row leave most of the chip idle (16 blocks of 64
+// x 128 on 2048 columns) and pay 0.4 us a stage.  One row / the tiles, us (weights
+// from memory): K 2048, 64 columns 8.6 / 12.9, 2048 9.0 / 13.9, 6144 9.4 / 14.0,
+// 16384 13.5 / 15.7, 20480 21.2 / 15.9; K 512, 2048 columns 3.9 / 5.8, 16384 5.4 /
+// 6.7, 32768 8.7 / 7.7; K 4096, 4096 columns 15.8 / 24.2, 16384 23.0 / 26.8, 24576
+// 38.6 / 30.3; K 8192, 8192 columns 31 / 46.  The rings let two blocks share a CU:
+// above 512 blocks the tiles are the faster form.
+constexpr int64_t ROW_MAX_N = 512 * RW_COLS;
+__global__ __launch_bounds__(64) void gemm_w8_row_kernel(const GemmArgs a) {
+  using Dot = RowDot<true, 1>;
+  __shared__ __align__(1024) uint8_t lds[Dot::LDS];
+  const int lane = threadIdx.x;
+  const int64_t n0 = (int64_t)blockIdx.x * RW_COLS, n = n0 + (lane & 31);
+  const int64_t m = a.x_rows ? (int64_t)a.x_rows[0] : 0;
+  const Dot d(lds, a.x + m * a.x_ld, 0, 1, reinterpret_cast<const int8_t*>(a.codes),
+              reinterpret_cast<const uint16_t*>(a.scale), (int)a.K, a.group,
+              [&](int c) { return n0 + c < a.N ? n0 + c : a.N - 1; });
+  uint16_t o = f2h(d.dot()[0]);
+  if (lane >= 32 || n >= a.N) return;
+  if (a.resid) o = hadd_round(h2f(o), a.resid[n]);
+  a.y16[n] = o;
+}
+
 // Block shapes: two blocks per CU each (at most 80 KB of LDS).
 template <class Q>
 using QWide = WideGeo<Q, 4, 2, 4, 2, Q::ZERO ? 16 : 32>;   // 128 x 256
@@ -307,6 +332,12 @@ TilePick tile_pick(int64_t M, int64_t N, bool row_out) {
 
 template <class Q, bool GATHERS>
 int launch_q(GemmArgs a, hipStream_t st) {
+  if constexpr (std::is_same_v<Q, WideW8>) {
+    if (a.M == 1 && a.N <= ROW_MAX_N) {
+      hipLaunchKernelGGL(gemm_w8_row_kernel, dim3((unsigned)((a.N + RW_COLS - 1) / RW_COLS)), dim3(64), 0, st, a);
+      LEMOQ_CHECK_LAUNCH();
+    }
+  }
   const int64_t ng = a.K / a.group;
   a.scale_vec = !std::is_same_v<Q, WideMx4> && ng % 8 == 0 && lemoq_aligned16(a.scale);
   const TilePick pick = tile_pick(a.M, a.N, a.row_out != 0);

@@ -29,4 +29,11 @@ __device__ __forceinline__ void dma16(uint32_t to, uint64_t addr) {
                : "s"(to), "v"(addr)
                : "m0", "memory");
 }
+// 64 lanes x 2 bytes from addr (per lane), zero-extended, to LDS at `to` + 4 lane.
+__device__ __forceinline__ void dma2(uint32_t to, uint64_t addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, off"
+               :
+               : "s"(to), "v"(addr)
+               : "m0", "memory");
+}
 #pragma clang diagnostic pop

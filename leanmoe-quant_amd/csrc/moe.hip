@@ -17,18 +17,6 @@
 //           fp16 residual add.
 // Every wave issues all of its weight loads (plus the activation slice)
 // before any arithmetic, with the lane layout of the dense GEMV (gemv.hip).
-//
-// The _dq forms run the same launches with the arithmetic of the multi-token
-// block (moe_prefill.hip): weights rounded to fp16 before the dots, fp16 gate,
-// up, silu and product, fp16 expert outputs times the fp16 routing weight,
-// added in fp16 in ascending expert order.  They serve the one row that the
-// last layer of a prefill needs: bound by the latency of two dependent weight
-// streams (34 and 17 MB), where the grouped GEMMs on 32-row fragments with one
-// live row are bound by their K loop: H 2048, F 1024, top 8 of 64, gate/up
-// 24.9 -> 9.0 us with the routing, down 15.6 -> 6.7 with the combine, and no
-// routing, sort and combine launches (4 + 5 + 4 us).
-#include <type_traits>
-
 #include "common.h"
 
 namespace {
@@ -48,8 +36,8 @@ struct GateUpArgs {
 };
 
 // PL = 0: ids given; PL > 0: routed from E <= 64*PL logits.
-template <int KCH, int R, int PL, bool EXACT, bool DQ>
-__device__ __forceinline__ void gate_up_body(const GateUpArgs& a) {
+template <int KCH, int R, int PL, bool EXACT>
+__global__ __launch_bounds__(256) void moe_gate_up_kernel(const GateUpArgs a) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int slot = blockIdx.y;
   int64_t e = 0;
@@ -109,8 +97,8 @@ __device__ __forceinline__ void gate_up_body(const GateUpArgs& a) {
   float g[R], u[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    g[r] = wave_sum(DQ ? w8_row_dot_dq<R, KCH>(tg, r, xc) : w8_row_dot<R, KCH>(tg, r, xc));
-    u[r] = wave_sum(DQ ? w8_row_dot_dq<R, KCH>(tu, r, xc) : w8_row_dot<R, KCH>(tu, r, xc));
+    g[r] = wave_sum(w8_row_dot<R, KCH>(tg, r, xc));
+    u[r] = wave_sum(w8_row_dot<R, KCH>(tu, r, xc));
   }
   if (lane < R) {
     float gv = g[0], uv = u[0];
@@ -123,28 +111,14 @@ __device__ __forceinline__ void gate_up_body(const GateUpArgs& a) {
     if (!ev) gv = uv = 0.0f;
     const int n = n0 + lane;
     if (n < F) {
-      if constexpr (DQ) {
-        const float gh = h2f(f2h(gv));
-        a.act[(int64_t)slot * F + n] = f2h(h2f(f2h(gh / (1.0f + expf(-gh)))) * h2f(f2h(uv)));
-      } else {
-        const float sig = 1.0f / (1.0f + expf(-gv));
-        a.act[(int64_t)slot * F + n] = f2h(gv * sig * uv);
-      }
+      const float sig = 1.0f / (1.0f + expf(-gv));
+      a.act[(int64_t)slot * F + n] = f2h(gv * sig * uv);
     }
   }
 }
 
-template <int KCH, int R, int PL, bool EXACT>
-__global__ __launch_bounds__(256) void moe_gate_up_kernel(const GateUpArgs a) {
-  gate_up_body<KCH, R, PL, EXACT, false>(a);
-}
-template <int KCH, int R, int PL, bool EXACT>
-__global__ __launch_bounds__(256) void moe_gate_up_dq_kernel(const GateUpArgs a) {
-  gate_up_body<KCH, R, PL, EXACT, true>(a);
-}
-
-template <int KCH, int R, bool EXACT, bool DQ>
-__device__ __forceinline__ void down_body(
+template <int KCH, int R, bool EXACT>
+__global__ __launch_bounds__(512) void moe_down_kernel(
     const uint16_t* __restrict__ act, const int8_t* __restrict__ codes,
     const uint16_t* __restrict__ scale, const int64_t* __restrict__ ids,
     const uint16_t* __restrict__ top_w, int top_k, int E, int H, int F, int group,
@@ -161,11 +135,6 @@ __device__ __forceinline__ void down_body(
 
   for (int slot = wave; slot < top_k; slot += 8) {
     const int64_t e = ids[slot];
-    int at = slot;  // its place in the sum
-    if constexpr (DQ) {  // ascending expert id, slot order among equal ids
-      const int64_t o = ids[lane < top_k ? lane : 0];
-      at = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < top_k && (o < e || (o == e && lane < slot))));
-    }
     const float wslot = h2f(top_w[slot]);
     XRaw<KCH> av;
     x_issue<KCH, EXACT>(av, act + (int64_t)slot * F, F, true, lane);
@@ -179,8 +148,8 @@ __device__ __forceinline__ void down_body(
     x_chunks<KCH>(av, xc);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const float v = wave_sum(DQ ? w8_row_dot_dq<R, KCH>(t, r, xc) : w8_row_dot<R, KCH>(t, r, xc));
-      if (lane == 0) part[at][r] = !ev ? 0.0f : DQ ? h2f(f2h(h2f(f2h(v)) * wslot)) : v * wslot;
+      const float v = wave_sum(w8_row_dot<R, KCH>(t, r, xc));
+      if (lane == 0) part[slot][r] = ev ? v * wslot : 0.0f;
     }
   }
   __syncthreads();
@@ -188,43 +157,12 @@ __device__ __forceinline__ void down_body(
     const int n = n0 + t;
     if (n < H) {
       float v = 0.0f;
-      for (int i = 0; i < top_k; ++i) v = DQ ? h2f(f2h(v + part[i][t])) : v + part[i][t];
+      for (int i = 0; i < top_k; ++i) v += part[i][t];
       uint16_t o = f2h(v);
       if (resid) o = hadd_round(h2f(o), res);
       out[n] = o;
     }
   }
-}
-
-template <int KCH, int R, bool EXACT>
-__global__ __launch_bounds__(512) void moe_down_kernel(
-    const uint16_t* __restrict__ act, const int8_t* __restrict__ codes,
-    const uint16_t* __restrict__ scale, const int64_t* __restrict__ ids,
-    const uint16_t* __restrict__ top_w, int top_k, int E, int H, int F, int group,
-    const uint16_t* __restrict__ resid, uint16_t* __restrict__ out) {
-  down_body<KCH, R, EXACT, false>(act, codes, scale, ids, top_w, top_k, E, H, F, group, resid, out);
-}
-template <int KCH, int R, bool EXACT>
-__global__ __launch_bounds__(512) void moe_down_dq_kernel(
-    const uint16_t* __restrict__ act, const int8_t* __restrict__ codes,
-    const uint16_t* __restrict__ scale, const int64_t* __restrict__ ids,
-    const uint16_t* __restrict__ top_w, int top_k, int E, int H, int F, int group,
-    const uint16_t* __restrict__ resid, uint16_t* __restrict__ out) {
-  down_body<KCH, R, EXACT, true>(act, codes, scale, ids, top_w, top_k, E, H, F, group, resid, out);
-}
-
-template <int KCH>
-int launch_gate_up_dq(hipStream_t st, const GateUpArgs& a) {  // routed from E <= 256 logits
-  constexpr int R = 2;
-  const dim3 grid((unsigned)((a.F + 4 * R - 1) / (4 * R)), (unsigned)a.top_k);
-  const bool exact = a.H == 1024 * KCH && a.F % (4 * R) == 0;
-  if (exact && a.E <= 64)
-    hipLaunchKernelGGL((moe_gate_up_dq_kernel<KCH, R, 1, true>), grid, dim3(256), 0, st, a);
-  else if (exact)
-    hipLaunchKernelGGL((moe_gate_up_dq_kernel<KCH, R, 4, true>), grid, dim3(256), 0, st, a);
-  else
-    hipLaunchKernelGGL((moe_gate_up_dq_kernel<KCH, R, 4, false>), grid, dim3(256), 0, st, a);
-  LEMOQ_CHECK_LAUNCH();
 }
 
 template <int KCH>
@@ -252,17 +190,10 @@ int launch_gate_up(hipStream_t st, const GateUpArgs& a, int pl) {
 template <int KCH>
 int launch_down(hipStream_t st, const uint16_t* act, const int8_t* codes, const uint16_t* scale,
                 const int64_t* ids, const uint16_t* top_w, int top_k, int E, int H, int F,
-                int group, const uint16_t* resid, uint16_t* out, bool dq) {
+                int group, const uint16_t* resid, uint16_t* out) {
   constexpr int R = 4;
   dim3 grid((unsigned)((H + R - 1) / R));
-  if (dq) {
-    if (F == 1024 * KCH && H % R == 0)
-      hipLaunchKernelGGL((moe_down_dq_kernel<KCH, R, true>), grid, dim3(512), 0, st, act, codes, scale,
-                         ids, top_w, top_k, E, H, F, group, resid, out);
-    else
-      hipLaunchKernelGGL((moe_down_dq_kernel<KCH, R, false>), grid, dim3(512), 0, st, act, codes, scale,
-                         ids, top_w, top_k, E, H, F, group, resid, out);
-  } else if (F == 1024 * KCH && H % R == 0)
+  if (F == 1024 * KCH && H % R == 0)
     hipLaunchKernelGGL((moe_down_kernel<KCH, R, true>), grid, dim3(512), 0, st, act, codes, scale,
                        ids, top_w, top_k, E, H, F, group, resid, out);
   else
@@ -332,11 +263,12 @@ extern "C" int lemoq_moe_gate_up_w8(const uint16_t* x, const int8_t* codes, cons
   return gate_up_dispatch(lemoq_stream(stream), a, 0);
 }
 
-namespace {
-
-int gate_up_routed(const uint16_t* x, const int8_t* codes, const uint16_t* scale, const uint16_t* router_logits,
-                   int64_t top_k, int norm_topk_prob, int64_t num_experts, int64_t ffn, int64_t hidden, int64_t group,
-                   uint16_t* act, int64_t* top_i, uint16_t* top_w, void* stream, bool dq) {
+extern "C" int lemoq_moe_gate_up_w8_routed(const uint16_t* x, const int8_t* codes,
+                                           const uint16_t* scale, const uint16_t* router_logits,
+                                           int64_t top_k, int norm_topk_prob,
+                                           int64_t num_experts, int64_t ffn, int64_t hidden,
+                                           int64_t group, uint16_t* act, int64_t* top_i,
+                                           uint16_t* top_w, void* stream) {
   int rc = check_gate_up(x, codes, scale, router_logits, act, top_k, num_experts, ffn, hidden,
                          group);
   if (rc) return rc;
@@ -348,18 +280,13 @@ int gate_up_routed(const uint16_t* x, const int8_t* codes, const uint16_t* scale
   a.norm = norm_topk_prob ? 1 : 0;
   a.ids_out = top_i;
   a.w_out = top_w;
-  if (!dq) return gate_up_dispatch(lemoq_stream(stream), a, num_experts <= 64 ? 1 : 4);
-  switch (kch_of(a.H)) {
-    case 1: return launch_gate_up_dq<1>(lemoq_stream(stream), a);
-    case 2: return launch_gate_up_dq<2>(lemoq_stream(stream), a);
-    case 4: return launch_gate_up_dq<4>(lemoq_stream(stream), a);
-    default: return launch_gate_up_dq<8>(lemoq_stream(stream), a);
-  }
+  return gate_up_dispatch(lemoq_stream(stream), a, num_experts <= 64 ? 1 : 4);
 }
 
-int moe_down(const uint16_t* act, const int8_t* codes, const uint16_t* scale, const int64_t* ids,
-             const uint16_t* top_w, int64_t top_k, int64_t num_experts, int64_t hidden, int64_t ffn, int64_t group,
-             const uint16_t* residual, uint16_t* out, void* stream, bool dq) {
+extern "C" int lemoq_moe_down_w8(const uint16_t* act, const int8_t* codes, const uint16_t* scale,
+                                 const int64_t* ids, const uint16_t* top_w, int64_t top_k,
+                                 int64_t num_experts, int64_t hidden, int64_t ffn, int64_t group,
+                                 const uint16_t* residual, uint16_t* out, void* stream) {
   if (!act || !codes || !scale || !ids || !top_w || !out) return LEMOQ_ERR_NULL;
   if (top_k <= 0 || top_k > 64 || num_experts <= 0 || ffn <= 0 || hidden <= 0)
     return LEMOQ_ERR_SHAPE;
@@ -367,50 +294,11 @@ int moe_down(const uint16_t* act, const int8_t* codes, const uint16_t* scale, co
     return LEMOQ_ERR_UNSUPPORTED;
   if (num_experts * hidden * ffn >= (int64_t)1 << 40) return LEMOQ_ERR_SHAPE;
   if (!lemoq_aligned16(codes) || !lemoq_aligned16(act)) return LEMOQ_ERR_ALIGN;
-  auto go = [&](auto kch) {
-    return launch_down<decltype(kch)::value>(lemoq_stream(stream), act, codes, scale, ids, top_w, (int)top_k,
-                                             (int)num_experts, (int)hidden, (int)ffn, (int)group, residual, out, dq);
-  };
+  hipStream_t st = lemoq_stream(stream);
   switch (kch_of(ffn)) {
-    case 1: return go(std::integral_constant<int, 1>{});
-    case 2: return go(std::integral_constant<int, 2>{});
-    case 4: return go(std::integral_constant<int, 4>{});
-    default: return go(std::integral_constant<int, 8>{});
+    case 1: return launch_down<1>(st, act, codes, scale, ids, top_w, (int)top_k, (int)num_experts, (int)hidden, (int)ffn, (int)group, residual, out);
+    case 2: return launch_down<2>(st, act, codes, scale, ids, top_w, (int)top_k, (int)num_experts, (int)hidden, (int)ffn, (int)group, residual, out);
+    case 4: return launch_down<4>(st, act, codes, scale, ids, top_w, (int)top_k, (int)num_experts, (int)hidden, (int)ffn, (int)group, residual, out);
+    default: return launch_down<8>(st, act, codes, scale, ids, top_w, (int)top_k, (int)num_experts, (int)hidden, (int)ffn, (int)group, residual, out);
   }
-}
-
-}  // namespace
-
-extern "C" int lemoq_moe_gate_up_w8_routed(const uint16_t* x, const int8_t* codes,
-                                           const uint16_t* scale, const uint16_t* router_logits,
-                                           int64_t top_k, int norm_topk_prob,
-                                           int64_t num_experts, int64_t ffn, int64_t hidden,
-                                           int64_t group, uint16_t* act, int64_t* top_i,
-                                           uint16_t* top_w, void* stream) {
-  return gate_up_routed(x, codes, scale, router_logits, top_k, norm_topk_prob, num_experts, ffn, hidden, group, act,
-                        top_i, top_w, stream, false);
-}
-
-extern "C" int lemoq_moe_gate_up_w8_routed_dq(const uint16_t* x, const int8_t* codes,
-                                              const uint16_t* scale, const uint16_t* router_logits,
-                                              int64_t top_k, int norm_topk_prob,
-                                              int64_t num_experts, int64_t ffn, int64_t hidden,
-                                              int64_t group, uint16_t* act, int64_t* top_i,
-                                              uint16_t* top_w, void* stream) {
-  return gate_up_routed(x, codes, scale, router_logits, top_k, norm_topk_prob, num_experts, ffn, hidden, group, act,
-                        top_i, top_w, stream, true);
-}
-
-extern "C" int lemoq_moe_down_w8(const uint16_t* act, const int8_t* codes, const uint16_t* scale,
-                                 const int64_t* ids, const uint16_t* top_w, int64_t top_k,
-                                 int64_t num_experts, int64_t hidden, int64_t ffn, int64_t group,
-                                 const uint16_t* residual, uint16_t* out, void* stream) {
-  return moe_down(act, codes, scale, ids, top_w, top_k, num_experts, hidden, ffn, group, residual, out, stream, false);
-}
-
-extern "C" int lemoq_moe_down_w8_dq(const uint16_t* act, const int8_t* codes, const uint16_t* scale,
-                                    const int64_t* ids, const uint16_t* top_w, int64_t top_k,
-                                    int64_t num_experts, int64_t hidden, int64_t ffn, int64_t group,
-                                    const uint16_t* residual, uint16_t* out, void* stream) {
-  return moe_down(act, codes, scale, ids, top_w, top_k, num_experts, hidden, ffn, group, residual, out, stream, true);
 }

@@ -220,6 +220,10 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
         _I,
         [_P, _P, _P, _P, _I64, _I, _I64, _I64, _I64, _I64, _P, _P, _P, _P],
     ),
+    "lemoq_moe_gate_up_w8_dq": (
+        _I,
+        [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P, _P],
+    ),
     "lemoq_moe_gate_up_w8_routed_dq": (
         _I,
         [_P, _P, _P, _P, _I64, _I, _I64, _I64, _I64, _I64, _P, _P, _P, _P],

@@ -19,7 +19,7 @@ sdpa causal attention  ``lemoq_attn_prefill_f16``; in the last layer only the la
                        query: ``lemoq_attn_split_f16`` + ``lemoq_attn_merge`` (nothing
                        after the last layer reads another position, so its
                        attention, o_proj, norm, router and MoE run on that row,
-                       in the ``_dq`` forms of the one-token launches)
+                       the MoE block in its one-row form, with the same bits)
 o_proj + residual      ``lemoq_gemm_w8`` with the residual in its epilogue
 post_attention norm    ``lemoq_prefill_norm_route`` (at most 64 experts, hidden a multiple
 router F.linear +      of 512 up to 2048), else ``lemoq_rmsnorm``, ``lemoq_gemm_f16_splitk``
@@ -123,6 +123,21 @@ def prefill_prompt(weights: Any, tokens: Any, kv: list, cos_tab: Any, sin_tab: A
     ybuf = torch.empty((pairs, H), **f16)
     qk_scale = float((1.0 / math.sqrt(D)) * LOG2E)
 
+    def norm_route(L: Any, rows: Any, n: int) -> None:
+        """xn = the post-attention norm of ``rows`` (n, H); top_w, top_i = their routing."""
+        norm = int(bool(s.norm_topk_prob))
+        if fused_route:  # the three launches below in one, the same bits
+            _hip.call("lemoq_prefill_norm_route", P(rows), n, H, P(L.ln_post), float(s.eps), P(L.router), E, K, norm,
+                      P(xn), P(top_w), P(top_i), st)
+            return
+        _hip.call("lemoq_rmsnorm", P(rows), n, H, P(L.ln_post), float(s.eps), P(xn), st)
+        if rsplit > 1:  # partials only; the routing launch sums them as the GEMM's finish would
+            _hip.call("lemoq_gemm_f16_splitk", P(xn), n, H, H, P(L.router), E, None, E, rsplit, P(rws), st)
+            _hip.call("lemoq_route_topk_splitk", P(rws), rsplit, n, E, K, norm, P(top_w), P(top_i), st)
+        else:
+            _hip.call("lemoq_gemm_f16_splitk", P(xn), n, H, H, P(L.router), E, P(rlog), E, 1, P(rws), st)
+            _hip.call("lemoq_route_topk", P(rlog), 1, n, E, E, K, norm, P(top_w), P(top_i), st)
+
     _hip.call("lemoq_gather_rows", P(weights.embed), s.vocab, H, P(tokens), T, P(h), st)
     _hip.call("lemoq_rmsnorm", P(h), T, H, P(weights.layers[0].ln_in), float(s.eps), P(xn), st)
     n_layers = len(weights.layers)
@@ -141,25 +156,13 @@ def prefill_prompt(weights: Any, tokens: Any, kv: list, cos_tab: Any, sin_tab: A
         if kv_f16 is not None:
             kv_f16.append((k16[:, :T].clone(), v16[:, :T].clone()))
         if li + 1 == n_layers and T > 1 and last_row_only:
-            _last_layer_last_row(L, T, q, k16, v16, h, xn, attn, rws, rsplit, rlog, top_w, top_i, pair_tok,
+            _last_layer_last_row(L, T, q, k16, v16, h, xn, attn, norm_route, top_w, top_i, pair_tok,
                                  pair_src, pair_w, expert_off, tiles, act, ybuf, s, S, qk_scale, lib, st)
             break
         _hip.call("lemoq_attn_prefill_f16", P(q), HD, P(k16), P(v16), S * D, T, NH, D, qk_scale, P(attn), HD, st)
         _hip.call("lemoq_gemm_w8", P(attn), T, HD, HD, None, P(L.o_codes), P(L.o_scale), H, g, P(h), H, P(h), H,
                   st)
-        if fused_route:  # the three launches below in one, the same bits
-            _hip.call("lemoq_prefill_norm_route", P(h), T, H, P(L.ln_post), float(s.eps), P(L.router), E, K,
-                      int(bool(s.norm_topk_prob)), P(xn), P(top_w), P(top_i), st)
-        elif rsplit > 1:  # partials only; the routing launch sums them as the GEMM's finish would
-            _hip.call("lemoq_rmsnorm", P(h), T, H, P(L.ln_post), float(s.eps), P(xn), st)
-            _hip.call("lemoq_gemm_f16_splitk", P(xn), T, H, H, P(L.router), E, None, E, rsplit, P(rws), st)
-            _hip.call("lemoq_route_topk_splitk", P(rws), rsplit, T, E, K, int(bool(s.norm_topk_prob)), P(top_w),
-                      P(top_i), st)
-        else:
-            _hip.call("lemoq_rmsnorm", P(h), T, H, P(L.ln_post), float(s.eps), P(xn), st)
-            _hip.call("lemoq_gemm_f16_splitk", P(xn), T, H, H, P(L.router), E, P(rlog), E, 1, P(rws), st)
-            _hip.call("lemoq_route_topk", P(rlog), 1, T, E, E, K, int(bool(s.norm_topk_prob)), P(top_w), P(top_i),
-                      st)
+        norm_route(L, h, T)
         _hip.call("lemoq_moe_prefill_sort", P(top_i), P(top_w), T, K, E, P(pair_tok), P(pair_src), P(pair_w),
                   P(expert_off), P(tiles), max_tiles, st)
         _hip.call("lemoq_moe_prefill_gate_up", P(xn), H, P(pair_tok), P(tiles), max_tiles, P(L.gu_codes),
@@ -194,8 +197,8 @@ def prefill_prompt(weights: Any, tokens: Any, kv: list, cos_tab: Any, sin_tab: A
     # after these kernels.
 
 
-def _last_layer_last_row(L: Any, T: int, q: Any, k16: Any, v16: Any, h: Any, xn: Any, attn: Any, rws: Any,
-                         rsplit: int, rlog: Any, top_w: Any, top_i: Any, pair_tok: Any, pair_src: Any, pair_w: Any,
+def _last_layer_last_row(L: Any, T: int, q: Any, k16: Any, v16: Any, h: Any, xn: Any, attn: Any, norm_route: Any,
+                         top_w: Any, top_i: Any, pair_tok: Any, pair_src: Any, pair_w: Any,
                          expert_off: Any, tiles: Any, act: Any, ybuf: Any, s: Any, S: int, qk_scale: float,
                          lib: Any, st: Any) -> None:
     """The last layer after its KV rows are written, for the last position only.
@@ -205,10 +208,9 @@ def _last_layer_last_row(L: Any, T: int, q: Any, k16: Any, v16: Any, h: Any, xn:
     already in the cache.  So the last layer's attention runs for the one query at
     T - 1 over keys 0..T-1 (the decode split-KV fp16 kernel and its merge, on the
     fp16 K/V rows the prologue just wrote), and o_proj + residual, the post norm,
-    the router and the MoE block run on that row: for the shapes that the one-token
-    launches of a decode step take, in their ``_dq`` forms (the other layers'
-    roundings, other fp32 summation orders), else with the same kernels as the
-    other layers.
+    the router and the MoE block run on that row, with the bits of the other
+    layers' launches (the MoE block in its one-row form, ``lemoq_moe_*_w8_dq``, or
+    in those launches themselves).
     """
     P = _hip.ptr
     H, NH, D, E, K, F = s.hidden, s.heads, s.head_dim, s.num_experts, s.top_k, s.ffn
@@ -223,31 +225,18 @@ def _last_layer_last_row(L: Any, T: int, q: Any, k16: Any, v16: Any, h: Any, xn:
     hl = h[T - 1:]
     _hip.call("lemoq_attn_split_f16", P(q[T - 1:]), P(k16), P(v16), S * D, P(filled), NH, D, ns, qk_scale, P(m),
               P(ls), P(acc), st)
-    norm = int(bool(s.norm_topk_prob))
-    if D == 128 and NH in (4, 8, 16, 32) and H in (2048, 4096) and E <= 256 and K <= min(8, E) and F <= 8192:
-        # H 2048, F 1024, 8 of 64 experts: 4 launches, 25 us of GPU time; the 9 below 85 us
-        part = torch.empty((NH // 4, H), dtype=torch.float32, device=dev)
-        hr = torch.empty((H,), dtype=torch.float16, device=dev)
-        rl = torch.empty((E,), dtype=torch.float16, device=dev)
-        wk = torch.empty((K,), dtype=torch.float16, device=dev)
-        _hip.call("lemoq_attn_merge_o_proj_w8_dq", P(m), P(ls), P(acc), NH, ns, D, P(L.o_codes), P(L.o_scale), H, g,
-                  P(part), st)
-        _hip.call("lemoq_router_logits_resid", P(part), NH // 4, P(hl), P(L.ln_post), float(s.eps), H, P(L.router), E,
-                  P(hr), P(xn), P(rl), st)
-        _hip.call("lemoq_moe_gate_up_w8_routed_dq", P(xn), P(L.gu_codes), P(L.gu_scale), P(rl), K, norm, E, F, H, g,
-                  P(act), P(top_i), P(wk), st)
-        _hip.call("lemoq_moe_down_w8_dq", P(act), P(L.dn_codes), P(L.dn_scale), P(top_i), P(wk), K, E, H, F, g, P(hr),
-                  P(hl), st)
-        return
     _hip.call("lemoq_attn_merge", P(m), P(ls), P(acc), NH, ns, D, P(attn), st)
     _hip.call("lemoq_gemm_w8", P(attn), 1, HD, HD, None, P(L.o_codes), P(L.o_scale), H, g, P(hl), H, P(hl), H, st)
-    _hip.call("lemoq_rmsnorm", P(hl), 1, H, P(L.ln_post), float(s.eps), P(xn), st)
-    if rsplit > 1:
-        _hip.call("lemoq_gemm_f16_splitk", P(xn), 1, H, H, P(L.router), E, None, E, rsplit, P(rws), st)
-        _hip.call("lemoq_route_topk_splitk", P(rws), rsplit, 1, E, K, norm, P(top_w), P(top_i), st)
-    else:
-        _hip.call("lemoq_gemm_f16_splitk", P(xn), 1, H, H, P(L.router), E, P(rlog), E, 1, P(rws), st)
-        _hip.call("lemoq_route_topk", P(rlog), 1, 1, E, E, K, norm, P(top_w), P(top_i), st)
+    norm_route(L, hl, 1)
+    if H >= 2048 and E <= 256 and K <= 8 and F <= 8192:
+        # two launches of 13 and 10 us (H 2048, F 1024, 8 of 64 experts) for the four
+        # below of 44; the same bits, so narrower rows may stay where they are
+        wk = torch.empty((K,), dtype=torch.float16, device=dev)
+        _hip.call("lemoq_moe_gate_up_w8_dq", P(xn), P(L.gu_codes), P(L.gu_scale), P(top_i), P(top_w), K, E, F, H, g,
+                  P(act), P(wk), st)
+        _hip.call("lemoq_moe_down_w8_dq", P(act), P(L.dn_codes), P(L.dn_scale), P(top_i), P(wk), K, E, H, F, g, P(hl),
+                  P(hl), st)
+        return
     mt = int(lib.lemoq_moe_prefill_max_tiles(K, E))
     _hip.call("lemoq_moe_prefill_sort", P(top_i), P(top_w), 1, K, E, P(pair_tok), P(pair_src), P(pair_w),
               P(expert_off), P(tiles), mt, st)
