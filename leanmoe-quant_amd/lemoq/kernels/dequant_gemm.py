@@ -272,7 +272,7 @@ def _separate_dense(x: Any, qweight: Any, scale: Any, zero: Any, *, group_size: 
     """Separate arm of the other formats: fp16 ``dequantized_weight``
     (``src/lemoq/quant/linear.py:365-395``), then ``F.linear`` in fp16 with fp32
     accumulation.  fp16 scales (E8M0 for MXFP4) run one matrix-core GEMM on the
-    codes (``lemoq_gemm_q``); fp32 scales, groups of 16, and the narrow outputs
+    codes (``lemoq_gemm_q``); fp32 scales, groups that it does not take, and the narrow outputs
     of ``_weight_first`` materialise the weight first (``lemoq_dequant_q``,
     ``lemoq_gemm_f16``), with the same result."""
     if residual is not None:
@@ -283,8 +283,10 @@ def _separate_dense(x: Any, qweight: Any, scale: Any, zero: Any, *, group_size: 
     _check_rows(x, padded_in, "dequant_gemm_separate")
     half = torch.uint8 if mxfp4 else torch.float16
     M, N = int(x.shape[0]), int(qweight.shape[0])
-    if (scale.dtype == half and (symmetric or zero.dtype == half) and int(group_size) % 32 == 0
-            and not _weight_first(fmt, M, N, padded_in)):
+    # lemoq_gemm_q's scale groups: whole stages of 64 for QFMT_W8 (symmetric codes that come
+    # with a zero tensor), whole chunks of 32 for the others
+    if (scale.dtype == half and (symmetric or zero.dtype == half)
+            and int(group_size) % (64 if fmt == QFMT_W8 else 32) == 0 and not _weight_first(fmt, M, N, padded_in)):
         # dequantised in registers, to the same fp16 weights (lemoq_gemm_q)
         y = torch.empty((M, N), dtype=torch.float16, device=x.device)
         _hip.require_rocm(x, qweight, scale, None if symmetric else zero, what="dequant_gemm_separate")
