@@ -279,7 +279,7 @@ def _separate_dense(x: Any, qweight: Any, scale: Any, zero: Any, *, group_size: 
         raise NotImplementedError("the dequantise-then-GEMM arm takes no residual")
     bits, padded_in, fmt = _check_format(qweight, scale, zero, group_size, bits, symmetric, mxfp4)
     if padded_in % 64 != 0:
-        raise NotImplementedError("the fp16 GEMM needs padded_in % 64 == 0, got %d" % padded_in)
+        raise NotImplementedError("the fp16 GEMM needs padded_in %% 64 == 0, got %d" % padded_in)
     _check_rows(x, padded_in, "dequant_gemm_separate")
     half = torch.uint8 if mxfp4 else torch.float16
     M, N = int(x.shape[0]), int(qweight.shape[0])
@@ -312,7 +312,7 @@ def linear_f16(x: Any, weight: Any, *, splits: int = 1) -> Any:
         raise ValueError("weight must be contiguous fp16 (N, K)")
     N, K = int(weight.shape[0]), int(weight.shape[1])
     if K % 64 != 0:
-        raise NotImplementedError("linear_f16 needs K % 64 == 0, got %d" % K)
+        raise NotImplementedError("linear_f16 needs K %% 64 == 0, got %d" % K)
     _check_rows(x, K, "linear_f16")
     M = int(x.shape[0])
     y = torch.empty((M, N), dtype=torch.float16, device=x.device)

@@ -203,7 +203,7 @@ class OlmoeW8Weights:
         if lm_head not in ("w8", "fp16"):
             raise ValueError("lm_head must be 'w8' or 'fp16', got %r" % (lm_head,))
         if bits == 4 and shape.group_size % 32 != 0:
-            raise ValueError("4-bit weights need group_size % 32 == 0, got %d" % shape.group_size)
+            raise ValueError("4-bit weights need group_size %% 32 == 0, got %d" % shape.group_size)
         dev = torch.device(device)
         _hip.require_rocm(torch.empty(0, device=dev), what="OlmoeW8Weights.random")
         gen = torch.Generator(device=dev)

@@ -58,3 +58,14 @@ def test_entry_takes_what_it_is_given(bits, symmetric, mxfp4, group, scale_dtype
     if in_gemm:
         fmt, g = calls[0][1][5], calls[0][1][9]
         assert fmt == formats.format_id(bits, symmetric, mxfp4) and g == group
+
+
+def test_refusals_of_a_half_stage_say_what_they_need(calls):
+    """2000 MXFP4 inputs pad to 2016, which is no multiple of 64: several tokens are refused."""
+    rows = torch.zeros((M, 2016), dtype=torch.float16)
+    q, scale = torch.zeros((N, 1008), dtype=torch.uint8), torch.ones((N, 63), dtype=torch.uint8)
+    with pytest.raises(NotImplementedError, match=r"padded_in % 64 == 0, got 2016"):
+        dg.dequant_gemm_separate(rows, q, scale, group_size=32, bits=4, mxfp4=True)
+    with pytest.raises(NotImplementedError, match=r"K % 64 == 0, got 2016"):
+        dg.linear_f16(rows, torch.zeros((N, 2016), dtype=torch.float16))
+    assert not calls
