@@ -43,6 +43,10 @@ def unavailable_reason() -> str | None:
 def fused_available() -> bool:
     """True when the HIP library is built and a ROCm device is visible (never raises)."""
     try:
+        # asked for on every call of a QuantLinear: a loaded library and an initialised
+        # device need no look at the file system and the driver (3 us)
+        if _hip.loaded() and torch.cuda.is_initialized():
+            return True
         return _hip.library_available() and bool(torch.cuda.is_available())
     except Exception:  # noqa: BLE001
         return False

@@ -42,12 +42,7 @@ import torch
 from torch import nn
 
 from lemoq import _hip
-from lemoq.kernels.dequant_gemm import (
-    dequant_gemm_fused,
-    dequant_gemm_separate,
-    fused_available,
-    unavailable_reason,
-)
+from lemoq.kernels import dequant_gemm as kernels
 
 __all__ = ["DEQUANT_MODES", "QuantLinear", "QuantizeReport", "SchemeSpec", "TARGET_RULES", "classify_linear",
            "dequant_activity", "parse_scheme", "quantize_model", "realized_bytes", "reset_dequant_counters",
@@ -267,7 +262,7 @@ class QuantLinear(nn.Module):
     @property
     def fused_available(self) -> bool:
         """Whether the fused arm can run here (the HIP library and a ROCm device); never raises."""
-        return fused_available()
+        return kernels.fused_available()
 
     def _fused_fallback_reason(self, x: Any) -> str | None:
         """Why this call cannot take the fused arm, as the reference words it
@@ -287,9 +282,8 @@ class QuantLinear(nn.Module):
             return "input_width_mismatch(%d!=%d)" % (width, self.in_features)
         if x.numel() // max(self.in_features, 1) != 1:
             return "multi_token"
-        # a loaded library and a device tensor are what fused_available asks for
-        if not _hip.loaded() and not self.fused_available:
-            return "kernel_unavailable(%s)" % (unavailable_reason() or "unknown")
+        if not self.fused_available:
+            return "kernel_unavailable(%s)" % (kernels.unavailable_reason() or "unknown")
         return None
 
     def forward(self, x: Any) -> Any:
@@ -301,16 +295,16 @@ class QuantLinear(nn.Module):
         zero = None if self.symmetric else self.zero
         reason = self._fused_fallback_reason(xq)
         if reason is None:
-            y = dequant_gemm_fused(flat, self.packed, self.scale, zero, group_size=self.group_size,
-                                   bits=self.weight_bits, symmetric=self.symmetric, out_dtype=x.dtype,
-                                   mxfp4=self.mxfp4)
+            y = kernels.dequant_gemm_fused(flat, self.packed, self.scale, zero, group_size=self.group_size,
+                                           bits=self.weight_bits, symmetric=self.symmetric, out_dtype=x.dtype,
+                                           mxfp4=self.mxfp4)
             self._counters["fused_calls"] += 1
         else:
             xs = flat
             if self.padded_in != self.in_features:  # padded columns: zero inputs add nothing
                 xs = torch.nn.functional.pad(xs, (0, self.padded_in - self.in_features))
-            y = dequant_gemm_separate(xs, self.packed, self.scale, zero, group_size=self.group_size,
-                                      bits=self.weight_bits, symmetric=self.symmetric, mxfp4=self.mxfp4)
+            y = kernels.dequant_gemm_separate(xs, self.packed, self.scale, zero, group_size=self.group_size,
+                                              bits=self.weight_bits, symmetric=self.symmetric, mxfp4=self.mxfp4)
             y = y if x.dtype == y.dtype else y.to(x.dtype)
             # counted once the arm has run (this build has no CPU arm: a CPU input raises above)
             if reason != "mode_is_separate":
