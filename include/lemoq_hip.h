@@ -872,9 +872,10 @@ int lemoq_moe_prefill_sort(const int64_t* top_i, const float* top_w, int64_t T, 
 
 /* act (pairs, F) = fp16(fp16(silu(g)) * u), g and u the fp16 outputs of
  * x[pair_tok] @ w^T for the expert's gate rows [0, F) and up rows [F, 2F)
- * (w8, w = fp16(code * scale)).  A table of a caller's own holds 0 in its
- * fourth column.  x (T, H) fp16; gu_codes (E, 2F, H) int8;
- * gu_scale (E, 2F, H/group) fp16.  H, F and group multiples of 64. */
+ * (w8, w = fp16(code * scale)).  The fourth column of the table's first row is a
+ * hint of how many rows are used, for the order of the blocks alone: any value
+ * will do.  x (T, H) fp16; gu_codes (E, 2F, H) int8; gu_scale (E, 2F, H/group)
+ * fp16.  H, F and group multiples of 64. */
 int lemoq_moe_prefill_gate_up(const uint16_t* x, int64_t H, const int32_t* pair_tok,
                               const int32_t* tiles, int64_t max_tiles, const int8_t* gu_codes,
                               const uint16_t* gu_scale, int64_t F, int64_t group, uint16_t* act,
