@@ -169,7 +169,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 // The other formats (4-bit, asymmetric, MXFP4) were dequantised to an fp16
 // weight first and then multiplied: 6144 x 2048 4-bit weights, 317 rows, 37.1
 // -> 18.1 us.
-template <class G, bool GATHER>
+template <class G, bool GATHER, bool FAR = false>
 __global__ __launch_bounds__(G::NT, 2) void gemm_q_kernel(const GemmArgs a) {
   constexpr int OP = G::BN + 8;  // pitch of the output tile that the idle ring holds at the end (fp16)
   __shared__ __align__(1024) uint8_t lds[G::LDS > G::BM * OP * 2 ? G::LDS : G::BM * OP * 2];
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(G::NT, 2) void gemm_q_kernel(const GemmArgs a) {
   const int64_t srow = (n0 + wrow(t % G::BN)) * ng;
   const WideScales<G> sc(reinterpret_cast<const Raw*>(a.scale) + srow, reinterpret_cast<const Raw*>(a.zero) + srow,
                          (int)ng, a.scale_vec);
-  WideSrc<G, GATHER> src;
+  WideSrc<G, GATHER, FAR> src;
 #pragma unroll
   for (int p = 0; p < G::XP; ++p) {
     const int r = wide_x_row<G>(p, wave, lane);
@@ -208,7 +208,10 @@ __global__ __launch_bounds__(G::NT, 2) void gemm_q_kernel(const GemmArgs a) {
 #pragma unroll
   for (int p = 0; p < G::CP; ++p) {
     const int r = wide_c_row<G>(p, wave, lane);
-    src.co[p] = (uint32_t)(wrow(r) * row_bytes) + wide_c_chunk<G>(r, lane);
+    if constexpr (FAR)
+      src.co[p] = (uint64_t)(uintptr_t)(src.cb + wrow(r) * row_bytes) + wide_c_chunk<G>(r, lane);
+    else
+      src.co[p] = (uint32_t)(wrow(r) * row_bytes) + wide_c_chunk<G>(r, lane);
   }
   int b_row0[G::FN];
 #pragma unroll
@@ -219,8 +222,8 @@ __global__ __launch_bounds__(G::NT, 2) void gemm_q_kernel(const GemmArgs a) {
 #pragma unroll
     for (int j = 0; j < G::FN; ++j) acc[i][j] = (f32x16){};
   wide_dispatch<G::MF>(nf, [&](auto nfc) {
-    wide_mainloop<G, decltype(nfc)::value, GATHER>(acc, src, (int)(a.K / BK), a.group / 32, lds, b_row0,
-                                                   [&](int g0) { sc.put(lds, g0); });
+    wide_mainloop<G, decltype(nfc)::value, GATHER, FAR>(acc, src, (int)(a.K / BK), a.group / 32, lds, b_row0,
+                                                        [&](int g0) { sc.put(lds, g0); });
   });
   if (a.row_out) {  // as gemm_kernel: through LDS (the idle ring), 16-byte chunks of whole rows
     constexpr int CPR = G::BN / 8, RPI = G::NT / CPR;
@@ -330,16 +333,27 @@ TilePick tile_pick(int64_t M, int64_t N, bool row_out) {
   return best;
 }
 
+constexpr int64_t NEAR_K = 1LL << 23;  // a tile's 256 rows of codes have 32-bit offsets
+
 template <class Q, bool GATHERS>
 int launch_q(GemmArgs a, hipStream_t st) {
   if constexpr (std::is_same_v<Q, WideW8>) {
-    if (a.M == 1 && a.N <= ROW_MAX_N) {
+    if (a.M == 1 && a.N <= ROW_MAX_N && a.K <= NEAR_K) {
       hipLaunchKernelGGL(gemm_w8_row_kernel, dim3((unsigned)((a.N + RW_COLS - 1) / RW_COLS)), dim3(64), 0, st, a);
       LEMOQ_CHECK_LAUNCH();
     }
   }
   const int64_t ng = a.K / a.group;
   a.scale_vec = !std::is_same_v<Q, WideMx4> && ng % 8 == 0 && lemoq_aligned16(a.scale);
+  if constexpr (std::is_same_v<Q, WideW8>) {
+    if (a.K > NEAR_K) {  // longer rows: 64-bit row addresses, one block shape
+      using G = QMid<Q>;
+      a.row_tiles = (int)((a.M + G::BM - 1) / G::BM);
+      hipLaunchKernelGGL((gemm_q_kernel<G, true, true>), dim3((unsigned)(a.row_tiles * ((a.N + G::BN - 1) / G::BN))),
+                         dim3(G::NT), 0, st, a);
+      LEMOQ_CHECK_LAUNCH();
+    }
+  }
   const TilePick pick = tile_pick(a.M, a.N, a.row_out != 0);
   a.row_tiles = (int)((a.M + pick.rows - 1) / pick.rows);
   // 64-bit row addresses for gathered rows, and for strides beyond a tile's 32-bit offsets
@@ -408,7 +422,6 @@ int check_gemm(const GemmArgs& a, int group_step = 64) {
   if (((a.M + 63) / 64) * ((a.N + 63) / 64) > 0x7fffffffLL) return LEMOQ_ERR_SHAPE;
   if (a.K % 64 != 0 || a.x_ld < a.K || a.x_ld % 8 != 0 || (a.y16 && a.y_ld < a.N)) return LEMOQ_ERR_SHAPE;
   if (a.codes && (a.group <= 0 || a.group % group_step != 0 || a.K % a.group != 0)) return LEMOQ_ERR_UNSUPPORTED;
-  if (a.codes && a.K > (1LL << 23)) return LEMOQ_ERR_SHAPE;  // a tile's codes are addressed by 32-bit offsets
   if (a.resid && a.resid_ld < a.N) return LEMOQ_ERR_SHAPE;
   if (a.splits < 1 || a.splits > 64 || a.K % (64LL * a.splits) != 0) return LEMOQ_ERR_SHAPE;
   if (a.splits > 1 && (!a.part || a.M * a.N > (1LL << 31)))
@@ -443,7 +456,7 @@ extern "C" int lemoq_gemm_q(const uint16_t* x, int64_t M, int64_t K, int64_t x_l
   const bool asym = fmt == LEMOQ_QFMT_W8_ASYM || fmt == LEMOQ_QFMT_W4_ASYM;
   if (!y || !qweight || (asym && !zero)) return LEMOQ_ERR_NULL;
   if (fmt == LEMOQ_QFMT_MXFP4 && group != 32) return LEMOQ_ERR_UNSUPPORTED;
-  if (x_ld >= (1LL << 22)) return LEMOQ_ERR_SHAPE;  // a tile's rows are addressed by 32-bit offsets
+  if (x_ld >= (1LL << 22) || K > NEAR_K) return LEMOQ_ERR_SHAPE;  // a tile's rows are addressed by 32-bit offsets
   GemmArgs a{};
   a.x = x; a.x_ld = x_ld; a.M = M; a.N = N; a.K = K;
   a.codes = reinterpret_cast<const uint8_t*>(qweight); a.scale = scale; a.zero = asym ? zero : nullptr;

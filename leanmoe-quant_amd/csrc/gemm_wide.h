@@ -134,13 +134,15 @@ struct WideGeo {
 };
 
 // A lane's sources: byte offsets from the (block-uniform) bases xb and cb, or,
-// for gathered X rows (GATHER), addresses in xo and no xb.
-template <class G, bool GATHER>
+// for gathered X rows (GATHER), addresses in xo and no xb; for rows too long for
+// 32-bit offsets (FAR, with GATHER) addresses in co too, and no cb.
+template <class G, bool GATHER, bool FAR = false>
 struct WideSrc {
+  static_assert(GATHER || !FAR, "far rows");
   const uint8_t* xb;
   const uint8_t* cb;
   std::conditional_t<GATHER, uint64_t, uint32_t> xo[G::XP];  // pass p: tile row 8 WN p + 8 wave + lane / 8
-  uint32_t co[G::CP];                                        // pass p: weight row wide_c_row
+  std::conditional_t<FAR, uint64_t, uint32_t> co[G::CP];     // pass p: weight row wide_c_row
 };
 
 // Tile row of this lane in pass p of the X / code loads, and the 16-byte
@@ -182,9 +184,10 @@ __device__ __forceinline__ void wide_wait() {
 // groups g0 .. g0 + MAXG - 1 to LDS: for g0 = 0 once the first loads are out,
 // then whenever a long K has used up the MAXG that fit.  On return no direct load is in
 // flight, and a barrier frees the LDS.
-template <class G, int NF, bool GATHER, class PutScales>
-__device__ __forceinline__ void wide_mainloop(f32x16 (&acc)[G::MF][G::FN], const WideSrc<G, GATHER>& src, int nst, int cpg,
-                                              uint8_t* lds, const int (&b_row0)[G::FN], const PutScales& put_scales) {
+template <class G, int NF, bool GATHER, bool FAR, class PutScales>
+__device__ __forceinline__ void wide_mainloop(f32x16 (&acc)[G::MF][G::FN], const WideSrc<G, GATHER, FAR>& src, int nst,
+                                              int cpg, uint8_t* lds, const int (&b_row0)[G::FN],
+                                              const PutScales& put_scales) {
   using Q = typename G::Q;
   constexpr int FN = G::FN, R = G::RING;
   constexpr int XP = (32 * NF + 8 * G::WN - 1) / (8 * G::WN), VM = XP + G::CP;  // loads per wave and stage
@@ -198,13 +201,19 @@ __device__ __forceinline__ void wide_mainloop(f32x16 (&acc)[G::MF][G::FN], const
     const uint32_t to = lds0 + (uint32_t)(buf * G::STAGE);
     if (p < XP) {
       const uint32_t row = to + (uint32_t)(8 * G::WN * p + 8 * wave) * 128u;
-      if constexpr (GATHER)
+      if constexpr (FAR)
+        dma16(row, src.xo[p] + (uint64_t)stage * (BK * 2));
+      else if constexpr (GATHER)
         dma16(row, src.xo[p] + (uint32_t)stage * (BK * 2));
       else
         dma16(row, src.xo[p], src.xb + (int64_t)stage * (BK * 2));
-    } else
-      dma16(to + (uint32_t)(G::XB + (G::CR * (p - XP) + 64 / G::LPR * wave) * G::RB), src.co[p - XP],
-            src.cb + (int64_t)stage * G::RB);
+    } else {
+      const uint32_t row = to + (uint32_t)(G::XB + (G::CR * (p - XP) + 64 / G::LPR * wave) * G::RB);
+      if constexpr (FAR)
+        dma16(row, src.co[p - XP] + (uint64_t)stage * G::RB);
+      else
+        dma16(row, src.co[p - XP], src.cb + (int64_t)stage * G::RB);
+    }
   };
   // the ring starts with stages 0 .. R - 1 (clamped: a re-read is harmless)
 #pragma unroll
