@@ -107,7 +107,9 @@ def prefill_prompt(weights: Any, tokens: Any, kv: list, cos_tab: Any, sin_tab: A
     # the router's 64 outputs give few output tiles: K is cut into up to 8 ranges
     # whose fp32 partials the routing launch sums; fp16 logits only without a split
     rsplit = next(sp for sp in (8, 4, 2, 1) if H % (64 * sp) == 0)
-    fused_route = rsplit == 8 and E <= 64 and H <= 2048 and K <= E
+    # lemoq_prefill_norm_route, unlike the norm kernel, takes 16-byte aligned norm weights only
+    fused_route = (rsplit == 8 and E <= 64 and H <= 2048 and K <= E
+                   and all(P(L.ln_post) % 16 == 0 for L in weights.layers))
     rlog = torch.empty((T, E), **f16) if rsplit == 1 else None
     rws = torch.empty((rsplit, T, E), dtype=torch.float32, device=dev)
     top_w = torch.empty((T, K), dtype=torch.float32, device=dev)
