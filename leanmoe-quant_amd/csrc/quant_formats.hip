@@ -746,12 +746,18 @@ __global__ __launch_bounds__(256) void rtn_q_kernel(const T* __restrict__ w, int
 // Needs cols % 8 == 0 and 16-byte aligned weights and codes.  Bound by memory:
 // each weight is read once and its code written once.
 //
-// The quotient w / s is formed with the group's reciprocal y = RN(1 / s): q =
-// RN(w y) lies within one ulp of w / s, and RN(q + RN(w - s q) y) is then the
-// correctly rounded quotient (Markstein's theorem; the residual is exact when
-// nothing under- or overflows), the same value as the IEEE division in three
-// instructions per weight.  Groups whose scale is near the ends of fp32's
-// range or that hold infinities divide as before.
+// The quotient x = w / s is formed with the group's reciprocal in three
+// instructions per weight: y = RN(1 / s), q = RN(w y), RN(q + RN(w - s q) y).  It is
+// the correctly rounded quotient, as the IEEE division's.  q lies within 1.5 ulp of
+// x: w y is off by the reciprocal's error, less than an ulp, and then rounded.
+// Where that is at most one ulp the last step rounds right by Markstein's theorem.
+// In general it rounds x + d with |d| < 2^-22 ulp (1.5 ulp times the relative errors
+// of the residual and of y), which is wrong only if a midpoint of two floats lies
+// between; beside a midpoint the first error is half an ulp, the theorem's case, or
+// one and a half, which takes a w among the three largest significands:
+// tests/test_oracle_rtn_quotient.py runs those against every s, and quotients
+// as near to midpoints as there are.  Groups whose scale is near the ends of fp32's
+// range (over- and underflow of the steps) or that hold infinities divide.
 //
 // One layer's experts of OLMoE (402,653,184 fp16 weights, 8 bits): fp32 copy +
 // one wave per group of 128 with 4-byte loads and 1-byte stores 1574 us, this

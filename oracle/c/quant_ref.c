@@ -194,3 +194,13 @@ void oracle_mxfp4(const float* w, int64_t rows, int64_t cols, uint8_t* codes, ui
     }
   }
 }
+
+/* n quotients w / s as rtn_q8_kernel (csrc/quant_formats.hip) forms them: the
+ * reciprocal of s, a product and one correction, each rounded once. */
+void oracle_rtn_quotients(const float* w, const float* s, int64_t n, float* q) {
+  for (int64_t i = 0; i < n; ++i) {
+    const float y = 1.0f / s[i];
+    const float p = w[i] * y;
+    q[i] = fmaf(fmaf(-s[i], p, w[i]), y, p);
+  }
+}

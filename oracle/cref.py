@@ -37,6 +37,8 @@ def load():
         lib.oracle_rtn.restype = None
         lib.oracle_mxfp4.argtypes = [P, I64, I64, P, P]
         lib.oracle_mxfp4.restype = None
+        lib.oracle_rtn_quotients.argtypes = [P, P, I64, P]
+        lib.oracle_rtn_quotients.restype = None
         lib.oracle_f32_to_f16.argtypes = [ctypes.c_float]
         lib.oracle_f32_to_f16.restype = ctypes.c_uint16
         _lib = lib
@@ -93,3 +95,10 @@ def mxfp4(w: np.ndarray):
     scales = np.zeros((rows, nblk), dtype=np.uint8)
     load().oracle_mxfp4(w.ctypes.data, rows, cols, codes.ctypes.data, scales.ctypes.data)
     return codes, scales
+
+
+def rtn_quotients(w: np.ndarray, s: np.ndarray) -> np.ndarray:
+    w, s = (np.ascontiguousarray(a, dtype=np.float32) for a in (w, s))
+    q = np.empty_like(w)
+    load().oracle_rtn_quotients(w.ctypes.data, s.ctypes.data, w.size, q.ctypes.data)
+    return q
