@@ -111,7 +111,7 @@ def prefill_prompt(weights: Any, tokens: Any, kv: list, cos_tab: Any, sin_tab: A
     fused_route = (rsplit == 8 and E <= 64 and H <= 2048 and K <= E
                    and all(P(L.ln_post) % 16 == 0 for L in weights.layers))
     rlog = torch.empty((T, E), **f16) if rsplit == 1 else None
-    rws = torch.empty((rsplit, T, E), dtype=torch.float32, device=dev)
+    rws = None if fused_route else torch.empty((rsplit, T, E), dtype=torch.float32, device=dev)
     top_w = torch.empty((T, K), dtype=torch.float32, device=dev)
     top_i = torch.empty((T, K), dtype=torch.int64, device=dev)
     pairs = T * K
