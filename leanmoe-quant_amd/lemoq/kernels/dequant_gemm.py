@@ -258,17 +258,35 @@ def _weight_first(fmt: int, M: int, N: int, K: int) -> bool:
 
     In the GEMM every row tile dequantises its weight columns anew, and a stage
     of K takes as long as that; with few columns there is little weight to write
-    and too few blocks to hide it under.  One launch / two, us (MXFP4, MI355X):
-    K 4096, 64 columns x 400 rows 33 / 28, 512 x 1500 36 / 30, 1001 x 400 36 /
-    34, 512 x 4096 39 / 44, 1536 x 400 36 / 36, 2048 x 400 36 / 40; K 2048, 64 x
-    400 18 / 17, 512 x 2500 21 / 22.  Many rows of unaligned columns, whose
-    2-byte stores cost the wide tiles most: K 2048, 1001 x 2500 33 / 29, 1500 x
-    2500 34 / 40, 1500 x 4096 51 / 42; K 1024, 1001 x 2500 20 / 19."""
+    and too few blocks to hide it under.  What the two save in GPU time has to
+    pay for their second call (about 10 us of host time), so K counts.  One
+    launch / two, us on the GPU (MI355X; 8-bit asymmetric, 4-bit asymmetric,
+    MXFP4):
+      columns x rows K 2048                    K 4096                    K 8192
+      64 x 400       17/16  19/17  18/17       31/27  35/28  33/28       59/45  66/46  63/46
+      512 x 1500     19/19  21/19  21/19       34/31  37/31  37/31       65/53  71/54  70/54
+      1024 x 400     18/18  20/19  20/19       33/32  36/34  36/33       61/54  68/57  68/58
+      1536 x 640     19/20  20/21  20/21       33/33  37/36  37/36       62/53  70/58  69/57
+      2048 x 317     19/21  20/22  20/22       34/36  36/40  36/40       63/58  69/62  68/62
+      1792 x 1792    27/36  27/37  27/36       48/65  46/66  47/64       90/132  90/136  89/134
+    Columns that are no multiple of 8 leave by 2-byte stores, which cost the
+    GEMM's wide tiles most, while the fp16 GEMM's tiles are few rounds of the CUs:
+      1001 x 2500    31/30  35/30  35/30       55/51  61/52  61/50       105/101  111/99  111/98
+      1501 x 1536    30/29  33/30  32/29       50/51  58/52  56/51       92/93  107/95  107/94
+      1027 x 1920    29/26  32/26  30/26       49/40  56/41  52/40       89/71  104/73  97/72
+      1751 x 1792    31/36  35/37  33/36       54/65  60/66  60/65       100/133  110/137  111/136
+    and again where its 128 x 128 tiles are one for each CU (2047 x 2048: 34/33
+    36/33  34/32 at K 2048, 115/100  121/100  119/95 at K 8192).  Over 2496 sizes of
+    64 to 2048 columns the rule is within 5% of the better of the two for all but
+    127 of them, most of these just above 3072 rows."""
     if fmt in (QFMT_W8, QFMT_W4):
         return False
-    if N % 8 and K >= 2048 and (M > 1792 and N <= 1024 or M > 3072 and N <= 2048):
-        return True
-    return K >= 3072 and N <= 1024 and M * N <= 7 << 18
+    if N % 8 and K >= 2048:
+        if M > 1792 and N <= 1024 or M > 3072 and N <= 2048:
+            return True
+        if 1024 < N <= 2048 and (15 << 17 < M * N <= 47 << 16 or -(-M // 128) * -(-N // 128) == 256):
+            return True
+    return K >= 3072 and N <= (1024 if K < 6144 else 2048) and M * N <= 7 << 18
 
 
 def _separate_dense(x: Any, qweight: Any, scale: Any, zero: Any, *, group_size: int, bits: int, symmetric: bool,

@@ -69,3 +69,18 @@ def test_refusals_of_a_half_stage_say_what_they_need(calls):
     with pytest.raises(NotImplementedError, match=r"K % 64 == 0, got 2016"):
         dg.linear_f16(rows, torch.zeros((N, 2016), dtype=torch.float16))
     assert not calls
+
+
+@pytest.mark.parametrize("m,n,k,first", [(1024, 1792, 6144, True), (1024, 1793, 6144, False), (1, 2048, 8192, True),
+                                         (1, 2048, 4096, False), (896, 2048, 6144, True), (897, 2048, 6144, False),
+                                         (1312, 1501, 2048, True), (1309, 1501, 2048, False), (2052, 1501, 2048, True),
+                                         (2053, 1501, 2048, False), (1700, 1501, 1024, False), (1700, 1504, 2048, False),
+                                         (1, 2056, 8192, False), (2048, 2047, 2048, True), (2049, 2047, 2048, False), (2048, 2048, 2048, False),
+                                         (2, 1024, 3072, True), (2, 1024, 2048, False)])
+def test_weight_first_lines(m, n, k, first):
+    """Both sides of each line of the rule for narrow outputs; never for the formats that
+    dequantise in packed fp16."""
+    for fmt in (formats.QFMT_W8_ASYM, formats.QFMT_W4_ASYM, formats.QFMT_MXFP4):
+        assert dg._weight_first(fmt, m, n, k) == first
+    for fmt in (formats.QFMT_W8, formats.QFMT_W4):
+        assert not dg._weight_first(fmt, m, n, k)
