@@ -1232,7 +1232,7 @@ def main(argv=None) -> int:
 # Launch order of one batched prefill (lemoq.model.prefill.prefill_prompt):
 # gather, layer 0's input norm, 15 x [9 launches] (each combine also writes the
 # next layer's input norm), the last layer (qkv and KV rows for every position,
-# then 5 launches on the last row), the lm_head GEMV of the last row
+# then 6 launches on the last row), the lm_head GEMV of the last row
 # (final norm in its prologue), then the greedy pick; each role with the
 # kernel-name fragment its dispatch must carry.
 PREFILL_HEAD_ROLES = (("gather_rows", "gather_rows_kernel"), ("rmsnorm (input, layer 0)", "rmsnorm_kernel"))
@@ -1246,10 +1246,11 @@ PREFILL_COMBINE_NORM = ("moe_prefill_combine (+residual, next input norm)", "moe
 PREFILL_LAST_LAYER_ROLES = (("gemm_w8 qkv", "gemm_q_kernel"),
                             ("qk_rows (q/k norm, RoPE, KV-INT8)", "qk_rows_kernel"),
                             ("last row: attention split-KV", "attn_split_kernel"),
-                            ("last row: attention merge + o_proj", "merge_oproj_dq_kernel"),
-                            ("last row: residual + post norm + router", "router_resid_kernel"),
-                            ("last row: routing + gate_up", "moe_gate_up_dq_kernel"),
-                            ("last row: down + combine (+residual)", "moe_down_dq_kernel"))
+                            ("last row: attention merge", "attn_merge"),
+                            ("last row: o_proj (+residual)", "gemm_w8_row_kernel"),
+                            ("last row: post norm + router + routing", "norm_route_kernel"),
+                            ("last row: gate_up", "moe_row_gate_up_kernel"),
+                            ("last row: down + combine (+residual)", "moe_row_down_kernel"))
 PREFILL_TAIL_ROLES = (("gemv_w8 lm_head (last row, + final norm)", "gemv_w8_kernel"),
                       ("argmax_advance", "argmax_advance_kernel"))
 

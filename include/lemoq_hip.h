@@ -433,7 +433,9 @@ int lemoq_attn_merge_o_proj_w8(const float* m, const float* l, const float* acc,
                                int64_t group, float* part, void* stream);
 /* lemoq_attn_merge_o_proj_w8 with the weights rounded to fp16 before the dot
  * (fp16(code * scale), the multi-token QuantLinear's arithmetic,
- * src/lemoq/quant/linear.py:471-480): the last row of a prefill. */
+ * src/lemoq/quant/linear.py:471-480), the partial sums in this launch's own fp32
+ * order; a prefill's last row takes lemoq_attn_merge and lemoq_gemm_w8, whose order
+ * is that of its other rows. */
 int lemoq_attn_merge_o_proj_w8_dq(const float* m, const float* l, const float* acc,
                                   int64_t heads, int64_t num_splits, int64_t head_dim,
                                   const int8_t* codes, const uint16_t* scale, int64_t N,

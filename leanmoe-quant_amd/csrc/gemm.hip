@@ -9,8 +9,9 @@
 // (v_pk_mul_f16).
 //
 // Tiling: w8 weights run on the direct-load main loop of gemm_wide.h, in one
-// of three block shapes chosen by how the tiles fill the CUs (tile_pick); fp16
-// weights on the register-staged pipeline of gemm_core.h.  Tiles are numbered
+// of three block shapes chosen by how the tiles fill the CUs (tile_pick), one row
+// of them on row_gemm.h's wave per 32 columns; fp16 weights on the
+// register-staged pipeline of gemm_core.h.  Tiles are numbered
 // n-major (consecutive tiles share the weight tile) and each XCD takes a
 // contiguous range of them.
 //
@@ -301,14 +302,17 @@ template <class Q>
 using QSmall = WideGeo<Q, 2, 1, 4, 4, Q::ZERO ? 16 : 32>;  // 64 x 128
 
 // The shape and rows per tile with the least estimated time: a tile that has
-// a CU to itself takes `one`, and every further tile of a CU adds `more`
-// (measured at K = 2048 on 6144 and 2048 columns, 1 to 4096 rows, us; the
-// ratios are what counts, both grow with K alike).  Few rows per tile cost
-// matrix work for the weights' dequantisation, many leave CUs idle.  Rows that
-// go out element by element (unaligned) cost every tile its 2-byte stores, the
-// wide tiles most: 4099 columns, K = 1024, 512 rows 17.1 us with the constants
-// of aligned rows, 15.1 with these; 1500 rows 26.1 / 24.2; 1001 columns, 2300
-// rows 17.2 / 16.3 (the register-staged tiles before: 15.5, 24.6, 16.6).
+// a CU to itself takes `one`, and every further tile of a CU adds `more`.  They
+// rank the shapes and predict no time: measured at K = 2048 with CUs to spare
+// (us), where a full round of 256 tiles takes longer (128 x 256: 40 us against 31)
+// in every shape, and the stores at the end do not grow with K as the loop does.
+// Few rows per tile cost matrix work for the weights' dequantisation, many leave
+// CUs idle.  Rows that go out element by element (unaligned) cost every tile its
+// 2-byte stores, the wide tiles most (one_e, more_e): 4099 columns, K = 1024, 512
+// rows 17.1 us with the constants of aligned rows, 15.1 with these; 1500 rows 26.1
+// / 24.2.  Of 198 sizes (K 1024, 2048, 4096; 1024 to 6144 columns, aligned or not;
+// 32 to 4096 rows) with all five candidates timed, the one picked is within 4% of
+// the best at 194; the others are 5, 7, 7 and 10% off (unaligned, 700 to 3000 rows).
 struct TilePick {
   int shape, rows;
 };

@@ -18,10 +18,9 @@ __global__ __launch_bounds__(256) void merge_oproj_kernel(const MergeOprojArgs a
   oproj_finish<NSMAX, false>(a, t, xs);
 }
 
-// The weights rounded to fp16 first (the multi-token o_proj's arithmetic): the
-// last row of a prefill, 4.7 us where a merge launch and a GEMM on 64-row tiles
-// with one live row took 4.4 + 15.4 (2048 x 2048, 16 heads; latency of one
-// weight stream against the GEMM's 32-stage K loop).
+// The weights rounded to fp16 first (the multi-token o_proj's roundings, in this
+// GEMV's fp32 order): 4.7 us for 2048 x 2048, 16 heads, where a merge and the one-row
+// GEMM, whose sums have the bits of the multi-token o_proj, take 4.5 + 10.1.
 template <int NSMAX>
 __global__ __launch_bounds__(256) void merge_oproj_dq_kernel(const MergeOprojArgs a) {
   __shared__ __align__(16) uint16_t xs[MO_COLS];
